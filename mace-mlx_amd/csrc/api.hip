@@ -104,6 +104,7 @@ struct Layer {
   DBuf<unsigned char> mlp_tiles_x;  // the same, split into fp16 pairs (float32 policy)
   float mlp_winv[3] = {1.f, 1.f, 1.f};
   float w3inv = 1.f;
+  int fold_exp[4] = {0, 0, 0, 0};  // first layer: exponents of the folded weights' largest magnitudes
   bool resid = true;       // residual block (skip from the input); else the skip acts on the message
   DBuf<float> mskip[4], mskipT[4], dens;
   int nskip = 0;
@@ -183,6 +184,19 @@ struct mace_ctx {
   // species z, the row maps of the per-species products
   DBuf<int> sp_perm;
   std::vector<int> sp_cnt, sp_off;
+  // First layer as neighbour sums (launch_first_fwd): the species present (ascending), their slots
+  // by species, and the folded weights' split planes per degree; nz = 0: not available (the loaded
+  // model or the species count)
+  struct FirstSum {
+    int nz = 0, kb = 0;
+    std::vector<int> present;
+    DBuf<int> zslot;  // slot by species [n_el], then the species present
+    DBuf<int> order;           // nz > 1: each receiver's edges by sender species (launch_first_order)
+    bool order_valid = false;  // order written for the current edge list and species
+    DBuf<_Float16> planes;  // folded weights: eight split matrices (degree, forward | VJP), one allocation
+    _Float16 *wf[4] = {}, *wb[4] = {};
+    bool edges_for = false;                // the edge buffers were laid out for this path
+  } first;
   DBuf<double> pos;
   double* pos_pinned = nullptr;
   size_t pos_pinned_n = 0;
@@ -431,6 +445,74 @@ void free_layers(mace_ctx* c) {
   c->layers.clear();
   for (auto& kv : c->wsplit) kv.second.x.release();
   c->wsplit.clear();
+  c->first.nz = 0;
+  c->first.present.clear();
+}
+
+// Exponents of the largest magnitudes of the first layer's folded weights over the model's elements
+// (the split planes' scales, one per degree)
+void measure_first_fold(mace_ctx* c) {
+  Layer& L = c->layers[0];
+  if (L.nonlin) return;
+  DBuf<unsigned> amax;
+  amax.ensure(4);
+  HIPCHK(hipMemset(amax.p, 0, 4 * sizeof(unsigned)));
+  const float* lin[4] = {L.lin_[0].p, L.lin_[1].p, L.lin_[2].p, L.lin_[3].p};
+  launch_first_fold(c->stream, L.wn, NC, L.mlp[3].p, c->up0_tab.p, nullptr, c->dims.num_elements, lin, nullptr, nullptr,
+                    nullptr, amax.p);
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipStreamSynchronize(c->stream));
+  unsigned m[4];
+  HIPCHK(hipMemcpy(m, amax.p, sizeof m, hipMemcpyDeviceToHost));
+  amax.release();
+  for (int lo = 0; lo < 4; ++lo) {
+    float f;
+    std::memcpy(&f, &m[lo], sizeof f);
+    L.fold_exp[lo] = f > 0.f && std::isfinite(f) ? std::ilogb(f) : 0;
+  }
+  const int nz = std::min<int>(c->dims.num_elements, kFirstMaxZ);
+  c->first.zslot.ensure(c->dims.num_elements + kFirstMaxZ);
+  c->first.planes.ensure((size_t)8 * 2 * 64 * nz * NC);
+}
+
+// The first layer's neighbour sums for the species now present (sp_cnt): slots and folded weights,
+// made again only when the set of species changed (before ensure_node_buffers, which sizes the
+// arrays the sums use).  Each species adds 64 columns to the node products, so more than
+// kFirstMaxZ of them take the general kernels; measured up to there, the sums are faster (steps of
+// the medium model on an fcc alloy of 2,048 atoms, 2 / 4 / 6 / 8 species: 1.28 / 1.27 / 1.30 / 1.34 ms
+// against 1.48 in float32, 1.04 / 1.05 / 1.07 / 1.09 against 1.20 in float16; 256 atoms:
+// 0.32 - 0.34 against 0.36).
+void set_first_sum(mace_ctx* c) {
+  auto& F = c->first;
+  Layer& L = c->layers[0];
+  std::vector<int> now;
+  for (int z = 0; z < (int)c->sp_cnt.size(); ++z)
+    if (c->sp_cnt[z] > 0) now.push_back(z);
+  if (L.nonlin || now.empty() || (int)now.size() > kFirstMaxZ) {
+    F.nz = 0;
+    return;
+  }
+  if (F.nz == 0 || now != F.present) {
+    const int nz = (int)now.size();
+    std::vector<int> tab(c->dims.num_elements + nz, 0);  // slot by species, then the species present
+    for (int k = 0; k < nz; ++k) tab[now[k]] = k, tab[c->dims.num_elements + k] = now[k];
+    HIPCHK(hipMemcpy(F.zslot.p, tab.data(), tab.size() * sizeof(int), hipMemcpyHostToDevice));
+    const float* lin[4];
+    float scale[4];
+    const size_t plane = (size_t)2 * 64 * nz * NC;
+    for (int lo = 0; lo < 4; ++lo) {
+      lin[lo] = L.lin_[lo].p;
+      scale[lo] = std::ldexp(1.f, 14 - L.fold_exp[lo]);
+      F.wf[lo] = F.planes.p + 2 * lo * plane;
+      F.wb[lo] = F.planes.p + (2 * lo + 1) * plane;
+    }
+    launch_first_fold(c->stream, L.wn, NC, L.mlp[3].p, c->up0_tab.p, F.zslot.p + c->dims.num_elements, nz, lin, F.wf,
+                      F.wb, scale, nullptr);
+    HIPCHK(hipGetLastError());
+    F.present = now;
+    F.nz = nz;
+    F.kb = first_blocks(nz);
+  }
 }
 
 // symmetric contraction, product linear and readout of layer l (both interaction kinds)
@@ -694,6 +776,7 @@ void build_model(mace_ctx* c) {
       }
     }
   }
+  measure_first_fold(c);
   c->max_lin = 1;
   for (const Layer& L : c->layers) c->max_lin = std::max(c->max_lin, L.tl());
   c->mts = (tp_table_entries(c->max_lin) + 15) / 16 * 16;
@@ -735,6 +818,7 @@ void ensure_node_buffers(mace_ctx* c) {
     c->zero_species.ensure(N);
     HIPCHK(hipMemset(c->zero_species.p, 0, (size_t)N * sizeof(int)));
   }
+  if (c->first.nz > 0) wmid = std::max(wmid, 16 * c->first.kb * NC);  // the first layer's sums S and dL/dS
   c->h[L].ensure((size_t)N * c->layers[L - 1].dhid);
   c->M.ensure((size_t)N * wmid);
   c->gM.ensure((size_t)N * wmid);
@@ -780,6 +864,9 @@ StepPath step_path(const mace_ctx* c) {
   return p;
 }
 
+// Layer l is the first layer evaluated as neighbour sums
+bool first_sum(const mace_ctx* c, size_t l) { return l == 0 && c->first.nz > 0 && step_path(c).fused; }
+
 // The fused VJP of layer L rebuilds w from h3 (half-precision policies, one or two input blocks,
 // standard interaction block), so its forward does not store w
 bool layer_rw(const mace_ctx* c, const Layer& L) {
@@ -787,7 +874,9 @@ bool layer_rw(const mace_ctx* c, const Layer& L) {
 }
 // layer l's h3 / h3inv: its own buffers when its VJP reads them and a later layer would overwrite
 // the shared ones
-bool own_h3(const mace_ctx* c, size_t l) { return l + 1 < c->layers.size() && layer_rw(c, c->layers[l]); }
+bool own_h3(const mace_ctx* c, size_t l) {
+  return l + 1 < c->layers.size() && !first_sum(c, l) && layer_rw(c, c->layers[l]);
+}
 float* h3_of(mace_ctx* c, size_t l) { return own_h3(c, l) ? c->layers[l].h3own.p : c->h3.p; }
 float* h3inv_of(mace_ctx* c, size_t l) { return own_h3(c, l) ? c->layers[l].h3invown.p : c->h3inv.p; }
 
@@ -797,10 +886,13 @@ void ensure_edge_buffers(mace_ctx* c, int64_t E) {
   int maxw = 0;
   const StepPath path = step_path(c);
   const bool half = path.h16;  // fp16 w / h3 / gw storage
+  c->first.edges_for = first_sum(c, 0);
+  c->first.order_valid = false;
+  if (c->first.edges_for && c->first.nz > 1) c->first.order.ensure(e);
   for (auto& ly : c->layers) {
     if (half)
       ly.wh.ensure(e * ly.wn);
-    else
+    else if (!first_sum(c, &ly - c->layers.data()))  // the neighbour sums need no per-edge weights
       ly.w.ensure(e * ly.wn);
     maxw = std::max(maxw, ly.wn);
     if (!path.split) ly.ds.ensure(e * 3 * RADIAL_H);
@@ -1185,6 +1277,7 @@ void run_gemm(mace_ctx* c, hipStream_t st, GemmGroup& g) {
     bool ok = true;
     for (int q = 0; q < g.n && ok; ++q) {
       GemmProb& P = g.p[q];
+      if (P.WX1) continue;  // the problem brings its planes
       auto a = c->wsplit.find(P.WT1);
       auto b = P.K2 > 0 ? c->wsplit.find(P.WT2) : a;
       ok = a != c->wsplit.end() && b != c->wsplit.end() && P.Cout % 64 == 0 && P.K1 % 32 == 0 && P.K2 % 32 == 0;
@@ -1314,7 +1407,15 @@ void check_step_path(const mace_ctx* c) {
     fail(MACE_ERR_UNSUPPORTED, "the %d-channel engine runs the fused split-product path only", NC);
 }
 
+// Also, once per edge list and species assignment, the order in which the first layer's neighbour
+// sums take each receiver's edges.
 void ensure_embed(mace_ctx* c) {
+  if (first_sum(c, 0) && c->first.nz > 1 && !c->first.order_valid) {
+    Site s(c, "first_order");
+    launch_first_order(c->stream, c->N, c->rowptr.p, c->sender.p, c->species.p, c->first.zslot.p, c->first.nz,
+                       c->first.order.p);
+    c->first.order_valid = true;
+  }
   if (c->embed_valid) return;
   Site s(c, "embed");
   launch_embed(c->stream, c->N, c->species.p, c->embed.p, c->layers[0].din, c->h[0].p, c->dims.feature_half,
@@ -1630,7 +1731,12 @@ void forward(mace_ctx* c, const double* pos, double* out, double* e_part) {
       forward_nonlin(c, (int)l, h, hn);
       continue;
     }
-    {
+    const bool sums = first_sum(c, l);
+    if (sums) {  // the hidden layers and the species-resolved sums of Y h3 over each receiver's edges
+      Site s(c, lname("first_sum", l));
+      launch_first_fwd(st, N, nb, c->rowptr.p, c->ef.p, c->Y.p, c->first.order.p, c->first.nz, c->first.kb,
+                       L.mlp_tiles_x.p, L.mlp_winv, c->M.p, half);
+    } else {
       Site s(c, lname("mlp_hidden", l));
       // split: h3 holds E x 2 x 64 fp16 (the same bytes as E x 64 floats)
       if (split)
@@ -1660,7 +1766,7 @@ void forward(mace_ctx* c, const double* pos, double* out, double* e_part) {
         g.p[g.n++] = gprob(N, 2 * b + 1, NC, NC, h, L.din, NC * b * b, 0, L.upT[b].p, L.h_up.p, L.din, NC * b * b, 0);
       run_gemm(c, st, g);
     }
-    {
+    if (!sums) {
       Site s(c, lname("tp_fwd", l));
       if (fused)
         launch_tpx_fwd(st, L.lin, N, E, c->rowptr.p, c->sender.p, c->Y.p, c->Mt.p, c->mts, h3_of(c, l),
@@ -1683,8 +1789,16 @@ void forward(mace_ctx* c, const double* pos, double* out, double* e_part) {
         int first, cnt;
         slot_range(L, lo, &first, &cnt);
         const int d = 2 * lo + 1;
-        g.p[g.n++] = gprob(N, d, cnt * NC, NC, c->M.p, L.dmid, NC * ao[first], NC * d, L.linT[lo].p, L.A.p, L.dint,
-                           NC * lo * lo, 0);
+        const int kb = c->first.kb;
+        if (sums) {
+          g.p[g.n++] = gprob(N, d, 64 * c->first.nz, NC, c->M.p, 16 * kb * NC, NC * kb * lo * lo, NC * d, nullptr,
+                             L.A.p, L.dint, NC * lo * lo, 0);
+          g.p[g.n - 1].WX1 = c->first.wf[lo];
+          g.p[g.n - 1].winv1 = std::ldexp(1.f, L.fold_exp[lo] - 14);
+        } else {
+          g.p[g.n++] = gprob(N, d, cnt * NC, NC, c->M.p, L.dmid, NC * ao[first], NC * d, L.linT[lo].p, L.A.p, L.dint,
+                             NC * lo * lo, 0);
+        }
         if (c->dims.density_norm) g.p[g.n - 1].rowscale = L.rinv.p;
       }
       run_gemm(c, st, g);
@@ -1746,7 +1860,8 @@ void backward(mace_ctx* c, bool stress, double* out, const double* e_part, doubl
   const bool h16 = path.h16, split = path.split, fused = path.fused;
   int gyp = NSLICE;  // dL/dY partials per edge
   if (fused)
-    for (const Layer& Ly : c->layers) gyp = std::max(gyp, tpx_parts(Ly.tl()));
+    for (size_t l = first_sum(c, 0) ? 1 : 0; l < c->layers.size(); ++l)
+      gyp = std::max(gyp, tpx_parts(c->layers[l].tl()));
   // dE/dh_L from the nonlinear readout: written by the forward's energy_readout pass
   float* gh = c->gh0.p;
   float* gh_next = c->gh1.p;
@@ -1790,14 +1905,31 @@ void backward(mace_ctx* c, bool stress, double* out, const double* e_part, doubl
         int first, cnt;
         slot_range(Ly, lo, &first, &cnt);
         const int d = 2 * lo + 1;
-        g.p[g.n++] = gprob(N, d, NC, cnt * NC, gmsg, Ly.dint, NC * lo * lo, 0, Ly.lin_[lo].p, c->gM.p, Ly.dmid,
-                           NC * ao[first], NC * d);
+        const int kb = c->first.kb;
+        if (first_sum(c, l)) {
+          g.p[g.n++] = gprob(N, d, NC, 64 * c->first.nz, gmsg, Ly.dint, NC * lo * lo, 0, nullptr, c->gM.p,
+                             16 * kb * NC, NC * kb * lo * lo, NC * d);
+          g.p[g.n - 1].WX1 = c->first.wb[lo];
+          g.p[g.n - 1].winv1 = std::ldexp(1.f, Ly.fold_exp[lo] - 14);
+        } else {
+          g.p[g.n++] = gprob(N, d, NC, cnt * NC, gmsg, Ly.dint, NC * lo * lo, 0, Ly.lin_[lo].p, c->gM.p, Ly.dmid,
+                             NC * ao[first], NC * d);
+        }
         if (c->dims.density_norm) g.p[g.n - 1].rowscale = Ly.rinv.p;
       }
       run_gemm(c, st, g);
     }
     const int first_edge_grad = (l == L - 1) ? 0 : 1;  // gY / gef: write on the first layer visited
-    if (fused) {
+    if (first_sum(c, l)) {  // dL/dS -> dL/dY and, through the hidden layers, dL/def
+      Site s(c, lname("first_sum_bwd", l));
+      int acc_gy = first_edge_grad;
+      if (!acc_gy && gyp > 1) {  // the other partials start at zero
+        launch_fill_zero(st, c->gY.p, E * 16 * gyp);
+        acc_gy = 1;
+      }
+      launch_first_bwd(st, N, nb, c->rowptr.p, c->ef.p, c->Y.p, c->first.order.p, c->first.nz, c->first.kb,
+                       Ly.mlp_tiles_x.p, Ly.mlp_winv, c->gM.p, c->gY.p, gyp, acc_gy, c->gef.p, first_edge_grad, half);
+    } else if (fused) {
       // dL/dw stays on chip: the radial-MLP output layer's VJP (dL/dh3 partials) is fused in
       Site s(c, lname("tp_bwd", l));
       int acc_gy = first_edge_grad;
@@ -1829,7 +1961,7 @@ void backward(mace_ctx* c, bool stress, double* out, const double* e_part, doubl
       else
         launch_mlp_gh3(st, E, Ly.wn, c->gw.p, Ly.mlp[3].p, c->h3.p, nullptr, nullptr);
     }
-    {
+    if (!first_sum(c, l)) {
       Site s(c, lname("mlp_hidden_bwd", l));
       if (split)
         launch_mlp_hidden_bwd_x(st, E, nb, Ly.mlp_tiles_x.p, Ly.mlp_winv, c->ef.p, nullptr, fused ? c->gh3p.p : c->h3.p,
@@ -1934,7 +2066,8 @@ static void free_all(mace_ctx* c) {
                   &c->node_e, &c->cutv, &c->gcut, &c->mh_dens, &c->gwb, &c->gP})
     b->release();
   c->zero_species.release();
-  for (auto* b : {&c->species, &c->sp_perm, &c->sender, &c->receiver, &c->shifts, &c->rowptr, &c->rowptr_s, &c->perm_s, &c->pos_s,
+  c->first.planes.release();
+  for (auto* b : {&c->species, &c->sp_perm, &c->first.zslot, &c->first.order, &c->sender, &c->receiver, &c->shifts, &c->rowptr, &c->rowptr_s, &c->perm_s, &c->pos_s,
                   &c->nl_img, &c->nl_img_s, &c->nl_cpre, &c->nl_hits, &c->nl_bin, &c->nl_bin_sorted, &c->nl_atoms, &c->nl_iota, &c->nl_counts,
                   &c->nl_bin_count, &c->nl_bin_start, &c->e_tmp_i, &c->e_tmp_j, &c->e_tmp_s, &c->e_perm,
                   &c->e_keys})
@@ -2011,6 +2144,7 @@ int mace_model_end(mace_ctx* c) {
     }
     if (c->system_ready) {
       set_species_order(c);
+      set_first_sum(c);
       ensure_node_buffers(c);
       ensure_edge_buffers(c, c->E);  // per-layer edge buffers of the new model
     }
@@ -2069,12 +2203,18 @@ void set_batch(mace_ctx* c, int32_t G, const int32_t* n_atoms, const int32_t* sp
   HIPCHK(hipMemcpy(c->gid.p, gid.data(), gid.size() * sizeof(int), hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(c->gcell.p, cells9, 9 * (size_t)G * sizeof(double), hipMemcpyHostToDevice));
   HIPCHK(hipMemset(c->gvir.p, 0, 9 * (size_t)G * sizeof(double)));
+  c->species_h.assign(species, species + n);
+  set_species_order(c);
+  set_first_sum(c);
   ensure_node_buffers(c);
   {
     c->species.ensure(std::max(n, 1));
     if (n > 0) HIPCHK(hipMemcpy(c->species.p, species, (size_t)n * sizeof(int), hipMemcpyHostToDevice));
-    c->species_h.assign(species, species + n);
-    set_species_order(c);
+    c->first.order_valid = false;
+    if (first_sum(c, 0) && (!c->first.edges_for || (c->first.nz > 1 && c->first.order.n < (size_t)c->E)))
+      ensure_edge_buffers(c, c->E);
+    else if (!first_sum(c, 0) && c->first.edges_for)
+      ensure_edge_buffers(c, c->E);
     if (topo_changed || c->edges_manual) {  // a manual edge list lasts until the next set_system
       c->nl_valid = false;
       c->edges_manual = false;

@@ -188,6 +188,29 @@ void launch_mlp_out_x(hipStream_t st, int64_t E, int W, const void* h3x, const f
 void launch_mlp_gh3(hipStream_t st, int64_t E, int W, const float* gw, const float* W3, float* gh3,
                     const float* b3, float* gwb);
 
+// First interaction layer as neighbour sums (scalar inputs that depend on the sender's species z
+// only; split products): S_z[n][lm][q] = sum over the edges of n from senders of species z of
+// Y[lm] h3[q], h3 = the radial MLP's last hidden activations of the edge.  nz species are present,
+// zslot[species] = 0 .. nz - 1; a node's row of S holds, per degree l, kb = first_blocks(nz) blocks
+// of [2l + 1][NC] with column 64 zslot + q running over the blocks.
+constexpr int kFirstMaxZ = 8;
+inline int first_blocks(int nz) { return (64 * nz + NC - 1) / NC; }
+// nz > 1: order[rowptr[n] + k] = the k-th edge of receiver n by its sender's species, as
+// zslot << 24 | (edge - rowptr[n])
+void launch_first_order(hipStream_t st, int N, const int* rowptr, const int* sender, const int* species,
+                        const int* zslot, int nz, int* order);
+void launch_first_fwd(hipStream_t st, int N, int nb, const int* rowptr, const float* ef, const float* Y,
+                      const int* order, int nz, int kb, const void* tiles, const float* winv3, float* S, int rnd);
+// gS (layout of S): partial 0 of the gyp dL/dY partials per edge and dL/def, written or added
+void launch_first_bwd(hipStream_t st, int N, int nb, const int* rowptr, const float* ef, const float* Y,
+                      const int* order, int nz, int kb, const void* tiles, const float* winv3, const float* gS,
+                      float* gY, int gyp, int accumulate_gY, float* gef, int accumulate, int rnd);
+// folded weights of the present species (or, with amax, the largest magnitude per degree over
+// species 0 .. nz - 1): see k_first_fold
+void launch_first_fold(hipStream_t st, int W, int cout, const float* W3, const float* x, const int* present, int nz,
+                       const float* const* lin, _Float16* const* wf, _Float16* const* wb, const float* scale,
+                       unsigned* amax);
+
 // mh-1 non-linear interaction block (blocks.py:611-807).  LayerNorm radial MLP (radial.py:344-357)
 // over [ef | source species embedding | target species embedding]: the species parts of the
 // first Linear are per-species tables ts / tt ([n_el][64], tt with the bias); tiles: the

@@ -1065,23 +1065,22 @@ __device__ __forceinline__ void layer64x(const h8 (*w)[4][NP][64], const float* 
   for (int t = 0; t < 4; ++t) acc[t] = d[t] * inv;
 }
 
-// forward of the split kernels: first layer over the Bessel features, then two 64-wide
+// forward of the split kernels for the lane's edge e (features zero unless live): first layer over the Bessel features, then two 64-wide
 // layers, the activations between them rounded by mode RND (the feature policy); dsp as in
 // hidden_fwd; leaves a1, a2, a3 (the VJP recomputes them this way, with the same
 // instructions, instead of reading saved derivatives)
 template <bool OPQ, int RND, int NP>
-__device__ __forceinline__ void hidden_fwd_x(const MlpFwdXT<NP>& sw, const float* winv, int64_t E, int64_t e0, int nb,
+__device__ __forceinline__ void hidden_fwd_x(const MlpFwdXT<NP>& sw, const float* winv, bool live, int64_t e, int nb,
                                              const float* __restrict__ ef, f4v* a1, f4v* a2, f4v* a3, float* dsp) {
   // half-precision policies: weights, features and activations are rounded values (zero lo
   // planes), so one product per operand pair
   constexpr bool FULL = RND == RND_NONE;
-  const int l = threadIdx.x & 63, r = l & 15, g = l >> 4;
-  const int64_t e = e0 + r;
+  const int g = (threadIdx.x & 63) >> 4;
   float x[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
     const int k = 8 * g + j;
-    x[j] = (e < E && k < nb) ? ef[e * nb + k] : 0.f;
+    x[j] = (live && k < nb) ? ef[e * nb + k] : 0.f;
   }
   {
     float inv;
@@ -1147,7 +1146,7 @@ __global__ void __launch_bounds__(64 * kHidFwdWaves) k_mlp_hidden_x(int64_t E, i
   for (int64_t gi = (int64_t)blockIdx.x * kHidFwdWaves + wv; gi < ngroups; gi += (int64_t)gridDim.x * kHidFwdWaves) {
     const int64_t e0 = gi * 16, e = e0 + r;
     f4v a1[4], a2[4], a3[4];
-    hidden_fwd_x<false, RND, NP>(sw, wi.w, E, e0, nb, ef, a1, a2, a3, (ds && e < E) ? ds + e * 3 * H + 4 * g : nullptr);
+    hidden_fwd_x<false, RND, NP>(sw, wi.w, e < E, e, nb, ef, a1, a2, a3, (ds && e < E) ? ds + e * 3 * H + 4 * g : nullptr);
     float v[16];
 #pragma unroll
     for (int q = 0; q < 16; ++q) v[q] = qh(silu(a3[q >> 2][q & 3]), RND);
@@ -1173,6 +1172,59 @@ __global__ void __launch_bounds__(64 * kHidFwdWaves) k_mlp_hidden_x(int64_t E, i
   }
 }
 
+// dL/def of the lane's edge (components k = 4g + i) from dL/dh3 (v, the lane's 16 features,
+// overwritten); dsl(k, out): silu' of layer k's pre-activations in the lane's layout
+template <bool OPQ, int RND, int NP, class DS>
+__device__ __forceinline__ f4v hidden_vjp(const MlpBwdXT<NP>& sw, const MlpWinv& wi, float* v, DS dsl) {
+  float dv[16];
+  f4v acc[4];
+  dsl(2, dv);
+#pragma unroll
+  for (int q = 0; q < 16; ++q) v[q] *= dv[q];
+  dsl(1, dv);
+  // the gradients are float32 (lo planes nonzero); the weights' lo planes are zero under a
+  // half-precision policy
+  constexpr bool WLO = RND == RND_NONE;
+  layer64x<OPQ, WLO, true, NP>(sw.w2T, v, wi.w[2], acc);
+#pragma unroll
+  for (int q = 0; q < 16; ++q) v[q] = acc[q >> 2][q & 3] * dv[q];
+  dsl(0, dv);
+  layer64x<OPQ, WLO, true, NP>(sw.w1T, v, wi.w[1], acc);
+#pragma unroll
+  for (int q = 0; q < 16; ++q) v[q] = acc[q >> 2][q & 3] * dv[q];
+  // g_ef = g_a1 W0^T: one output tile (rows k < nb)
+  float inv;
+  const float sc = edge_scale<16>(v, &inv);
+  inv *= wi.w[0];
+  f4v o = f4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    h8 xh, xl;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      _Float16 hi, lo;
+      split_pair(v[4 * (2 * c + (j >> 2)) + (j & 3)] * sc, hi, lo);
+      xh[j] = hi;
+      xl[j] = lo;
+    }
+    const int lo = lane_opaque<OPQ>();
+    const h8 wh = sw.w0T[c][0][lo];
+    if constexpr (WLO) o = mfma16h(sw.w0T[c][NP - 1][lo], xh, o);
+    o = mfma16h(wh, xl, o);
+    o = mfma16h(wh, xh, o);
+  }
+  return o * inv;
+}
+
+// the lane's components k = 4g + i < nb of one edge's dL/def row
+__device__ __forceinline__ void store_gef(float* row, int g, int nb, const f4v& o, int accumulate) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int k = 4 * g + i;
+    if (k < nb) row[k] = accumulate ? row[k] + o[i] : o[i];
+  }
+}
+
 // gh3: np partials [np][E][64] (stride pstride floats), added in order.  RECOMP:
 // silu'(a1..a3) from the forward layers recomputed from ef (tiles ftiles, rounding mode
 // RND as the forward) instead of read from ds.
@@ -1194,9 +1246,8 @@ __global__ void __launch_bounds__(64 * NW) k_mlp_hidden_bwd_x(int64_t E, int nb,
   for (int64_t gi = (int64_t)blockIdx.x * NW + wv; gi < ngroups; gi += (int64_t)gridDim.x * NW) {
     const int64_t e0 = gi * 16, e = e0 + r, ec = e < E ? e : E - 1;  // rows past the end: computed, not stored
     float v[16], dv[16];
-    f4v acc[4];
     f4v a1[4], a2[4], a3[4];  // RECOMP: the pre-activations, rebuilt
-    if constexpr (RECOMP) hidden_fwd_x<true, RND, NP>(swf, wi.w, E, e0, nb, ef, a1, a2, a3, nullptr);
+    if constexpr (RECOMP) hidden_fwd_x<true, RND, NP>(swf, wi.w, e < E, e, nb, ef, a1, a2, a3, nullptr);
     // silu' of layer k's pre-activations in the lane's layout (feature 16t + 4g + i -> [4t + i])
     auto dsl = [&](int k, float* out) {
       if constexpr (RECOMP) {
@@ -1213,51 +1264,294 @@ __global__ void __launch_bounds__(64 * NW) k_mlp_hidden_bwd_x(int64_t E, int nb,
 #pragma unroll
       for (int q = 0; q < 16; ++q) v[q] += dv[q];
     }
-    dsl(2, dv);
+    const f4v o = hidden_vjp<RECOMP, RND, NP>(sw, wi, v, dsl);
+    if (e < E) store_gef(gef + e * nb, g, nb, o, accumulate);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// First interaction layer (scalar input features): its conv-TP input x[sender] depends on the
+// sender's species z alone, so the sum over a receiver's edges factors as
+//   M[n][lm][u] = sum_z x_z[u] sum_q W3[q][l u] S_z[n][lm][q],
+//   S_z[n][lm][q] = sum over the edges e of n with a sender of species z of Y[e][lm] h3[e][q].
+// The radial MLP's output layer (64 x 512 products per edge in the general kernels) then acts once
+// per node and species instead of once per edge, folded with x_z and the message linear into the
+// weights of one grouped product (k_first_fold); M, the TP weights w and dL/dh3 of this layer never
+// exist.
+//
+// Forward: a block of four waves walks a contiguous range of receivers in 16-edge tiles, four per
+// step (each wave the hidden layers of one tile, h3 and Y left in LDS); then wave t adds the step's
+// tiles to columns q = 16t .. 16t + 15 of the current S_z[16 lm][64 q], a product with K = the
+// tile's edges (fp32 matrix cores; fp16 / bf16 ones under the half policies, whose Y and h3 are
+// such values), accumulated in float32 in edge order and written when the species or the receiver
+// changes: one accumulator tile per wave, whatever the species count.  A row's edges are taken in
+// the order of their sender's species (k_first_order), so a tile spans few species.
+// VJP: dL/dh3[e] = gS_z Y[e] and dL/dY[e] = gS_z^T h3[e] (K = 16 and K = 64, fp32 matrix cores) with
+// h3 recomputed, then the hidden layers' VJP in the same registers.
+// ---------------------------------------------------------------------------
+constexpr int kFirstRS = 80, kFirstYS = 16;  // LDS row strides (floats): the rows g of a step on distinct banks
+
+// position of S_z[lm][0] in a node's row of S: blocks of NC columns (64 zi + q), laid out as the
+// input of a grouped product over rows (node, m) of each degree
+__device__ __forceinline__ int first_col(int lm, int zi, int kb) {
+  const int l = lm < 1 ? 0 : lm < 4 ? 1 : lm < 9 ? 2 : 3, c = 64 * zi;
+  return NC * (kb * l * l + (c / NC) * (2 * l + 1) + lm - l * l) + c % NC;
+}
+
+// order[rowptr[n] + k] = z << 24 | (e - rowptr[n]): the edges of receiver n by the species slot z of
+// their sender, otherwise in order; one wave per receiver
+__global__ void __launch_bounds__(256) k_first_order(int N, const int* __restrict__ rowptr,
+                                                     const int* __restrict__ sender, const int* __restrict__ species,
+                                                     const int* __restrict__ zslot, int nz, int* __restrict__ order) {
+  const int n = blockIdx.x * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;
+  if (n >= N) return;  // whole wave
+  const int beg = rowptr[n], deg = rowptr[n + 1] - beg;
+  int zr[4];  // the first 256 edges' slots
 #pragma unroll
-    for (int q = 0; q < 16; ++q) v[q] *= dv[q];
-    dsl(1, dv);
-    // the gradients are float32 (lo planes nonzero); the weights' lo planes are zero under a
-    // half-precision policy
-    constexpr bool WLO = RND == RND_NONE;
-    layer64x<RECOMP, WLO, true, NP>(sw.w2T, v, wi.w[2], acc);
+  for (int c = 0; c < 4; ++c) zr[c] = 64 * c + l < deg ? zslot[species[sender[beg + 64 * c + l]]] : -1;
+  int at = beg;
+  for (int z = 0; z < nz; ++z) {
+    auto place = [&](int c, int zc) {
+      const unsigned long long m = __ballot(zc == z);
+      if (zc == z) order[at + __popcll(m & ((1ull << l) - 1))] = z << 24 | (64 * c + l);
+      at += __popcll(m);
+    };
 #pragma unroll
-    for (int q = 0; q < 16; ++q) v[q] = acc[q >> 2][q & 3] * dv[q];
-    dsl(0, dv);
-    layer64x<RECOMP, WLO, true, NP>(sw.w1T, v, wi.w[1], acc);
+    for (int c = 0; c < 4; ++c) place(c, zr[c]);
+    for (int c = 4; 64 * c < deg; ++c) place(c, 64 * c + l < deg ? zslot[species[sender[beg + 64 * c + l]]] : -1);
+  }
+}
+
+typedef short s4 __attribute__((ext_vector_type(4)));
+
+// acc += A B over K = 16 edges: the lane's A[row r][edge 4s + g] and B[edge 4s + g][column r]
+template <int RND>
+__device__ __forceinline__ f4v mfma_edges(const float* a, const float* b, f4v acc) {
+  if constexpr (RND == RND_F16) {
+    h4 x, y;
 #pragma unroll
-    for (int q = 0; q < 16; ++q) v[q] = acc[q >> 2][q & 3] * dv[q];
-    // g_ef = g_a1 W0^T: one output tile (rows k < nb)
-    float inv;
-    const float sc = edge_scale<16>(v, &inv);
-    inv *= wi.w[0];
-    f4v o = f4v{0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < 4; ++s) x[s] = (_Float16)a[s], y[s] = (_Float16)b[s];  // exact: fp16 values
+    return __builtin_amdgcn_mfma_f32_16x16x16f16(x, y, acc, 0, 0, 0);
+  } else if constexpr (RND == RND_BF16) {
+    s4 x, y;
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      h8 xh, xl;
+    for (int s = 0; s < 4; ++s) x[s] = (short)(__float_as_uint(a[s]) >> 16), y[s] = (short)(__float_as_uint(b[s]) >> 16);
+    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(x, y, acc, 0, 0, 0);  // exact: bf16 values
+  } else {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        _Float16 hi, lo;
-        split_pair(v[4 * (2 * c + (j >> 2)) + (j & 3)] * sc, hi, lo);
-        xh[j] = hi;
-        xl[j] = lo;
-      }
-      const int lo = lane_opaque<RECOMP>();
-      const h8 wh = sw.w0T[c][0][lo];
-      if constexpr (WLO) o = mfma16h(sw.w0T[c][NP - 1][lo], xh, o);
-      o = mfma16h(wh, xl, o);
-      o = mfma16h(wh, xh, o);
+    for (int s = 0; s < 4; ++s) acc = mfma16(a[s], b[s], acc);
+    return acc;
+  }
+}
+
+// MULTI: more than one species (order set)
+template <int RND, bool MULTI>
+__global__ void __launch_bounds__(256) k_first_fwd(int N, int nb, const int* __restrict__ rowptr,
+                                                   const float* __restrict__ ef, const float* __restrict__ Y,
+                                                   const int* __restrict__ order, int nz, int kb,
+                                                   const MlpFwdX* __restrict__ tiles, MlpWinv wi,
+                                                   float* __restrict__ S) {
+  constexpr int NP = RND == RND_NONE ? 2 : 1;
+  __shared__ MlpFwdXT<NP> sw;
+  __shared__ __align__(16) float sT[4][16 * kFirstRS];
+  __shared__ __align__(16) float sY[4][16 * kFirstYS];
+  __shared__ int sZ[4][16];
+  stage_planes<NP>(sw, tiles);
+  __syncthreads();
+  const int wv = threadIdx.x >> 6, l = threadIdx.x & 63, r = l & 15, g = l >> 4;
+  const int64_t ld = (int64_t)16 * kb * NC;
+  const int n1 = (int)((int64_t)N * (blockIdx.x + 1) / gridDim.x);
+  int n = (int)((int64_t)N * blockIdx.x / gridDim.x);  // cursor over the block's tiles: receiver,
+  if (n >= n1) return;                                 // its row and the next tile's start
+  int beg = rowptr[n], end = rowptr[n + 1], e0 = beg;
+  f4v acc = f4v{0.f, 0.f, 0.f, 0.f};
+  int zc = 0;  // species the accumulator belongs to
+  while (n < n1) {  // uniform over the block
+    // the step's four tiles (every receiver has at least one, so that empty rows write zeros)
+    int tn[4], tb[4], te[4], cnt[4];
+    bool last[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      tn[j] = n, tb[j] = beg, te[j] = e0;
+      cnt[j] = n < n1 ? min(end - e0, 16) : -1;
+      e0 += 16;
+      last[j] = e0 >= end;
+      if (n < n1 && last[j] && ++n < n1) e0 = beg = end, end = rowptr[n + 1];
     }
-    if (e < E) {
+    // tile wv: hidden layers, h3 and Y into LDS
+    int mb = tb[0], me = te[0], mc = cnt[0];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int k = 4 * g + i;
-        if (k < nb) {
-          float* dst = gef + e * nb + k;
-          *dst = accumulate ? *dst + o[i] * inv : o[i] * inv;
+    for (int j = 1; j < 4; ++j)
+      if (wv == j) mb = tb[j], me = te[j], mc = cnt[j];
+    if (mc >= 0) {
+      const bool live = r < mc;
+      int e = me + r, z = 0;
+      if constexpr (MULTI) {
+        const int o = live ? order[e] : 0;
+        e = mb + (o & 0xffffff), z = o >> 24;
+        if (g == 0) sZ[wv][r] = live ? z : -1;
+      }
+      *reinterpret_cast<float4*>(&sY[wv][r * kFirstYS + 4 * g]) =
+          live ? ld4(Y + (int64_t)e * 16 + 4 * g) : float4{0.f, 0.f, 0.f, 0.f};
+      f4v a1[4], a2[4], a3[4];
+      hidden_fwd_x<true, RND, NP>(sw, wi.w, live, e, nb, ef, a1, a2, a3, nullptr);
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        *reinterpret_cast<float4*>(&sT[wv][r * kFirstRS + 16 * t + 4 * g]) =
+            float4{qh(silu(a3[t][0]), RND), qh(silu(a3[t][1]), RND), qh(silu(a3[t][2]), RND), qh(silu(a3[t][3]), RND)};
+    }
+    __syncthreads();
+    // columns 16 wv .. + 15 of every tile's receiver
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (cnt[j] < 0) continue;
+      float y[4], h[4];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        y[s] = sY[j][(4 * s + g) * kFirstYS + r];
+        h[s] = sT[j][(4 * s + g) * kFirstRS + 16 * wv + r];
+      }
+      float* out = S + tn[j] * ld + 16 * wv + r;
+      auto flush = [&] {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) out[first_col(4 * g + i, zc, kb)] = acc[i];
+        acc = f4v{0.f, 0.f, 0.f, 0.f};
+      };
+      if constexpr (!MULTI) {
+        acc = mfma_edges<RND>(y, h, acc);
+        if (last[j]) flush();
+      } else {
+        if (cnt[j] > 0) {
+          int zs[4];
+#pragma unroll
+          for (int s = 0; s < 4; ++s) zs[s] = sZ[j][4 * s + g];
+          const int z0 = __builtin_amdgcn_readfirstlane(sZ[j][0]);
+          const int z1 = __builtin_amdgcn_readfirstlane(sZ[j][cnt[j] - 1]);
+          for (int z = z0; z <= z1; ++z) {
+            for (; zc < z; ++zc) flush();
+            float ym[4];
+#pragma unroll
+            for (int s = 0; s < 4; ++s) ym[s] = zs[s] == z ? y[s] : 0.f;
+            acc = mfma_edges<RND>(ym, h, acc);
+          }
+        }
+        if (last[j]) {
+          for (; zc < nz; ++zc) flush();
+          zc = 0;
         }
       }
     }
+    __syncthreads();
+  }
+}
+
+// VJP of the first layer's sums: gS (the layout of S) -> dL/dY (partial 0 of gyp per edge, written
+// or added) and dL/def; 1 << wl waves per receiver, each taking every (1 << wl)-th tile
+template <int RND, bool MULTI>
+__global__ void __launch_bounds__(256) k_first_bwd(int N, int wl, int nb, const int* __restrict__ rowptr,
+                                                   const float* __restrict__ ef, const float* __restrict__ Y,
+                                                   const int* __restrict__ order, int kb,
+                                                   const MlpFwdX* __restrict__ ftiles,
+                                                   const MlpBwdX* __restrict__ tiles, MlpWinv wi,
+                                                   const float* __restrict__ gS, float* __restrict__ gY, int gyp,
+                                                   int accumulate_gY, float* __restrict__ gef, int accumulate) {
+  constexpr int NP = RND == RND_NONE ? 2 : 1;
+  __shared__ MlpBwdXT<NP> sw;
+  __shared__ MlpFwdXT<NP> swf;
+  stage_planes<NP>(sw, tiles);
+  stage_planes<NP>(swf, ftiles);
+  __syncthreads();
+  const int wv = threadIdx.x >> 6, l = threadIdx.x & 63, r = l & 15, g = l >> 4;
+  const int wpr = 1 << wl, rpb = 4 >> wl, part = wv & (wpr - 1), sub = wv >> wl;
+  const int64_t ld = (int64_t)16 * kb * NC;
+  for (int n = blockIdx.x * rpb + sub; n < N; n += gridDim.x * rpb) {
+    const int beg = __builtin_amdgcn_readfirstlane(rowptr[n]), end = __builtin_amdgcn_readfirstlane(rowptr[n + 1]);
+    const float* gs = gS + n * ld;
+    for (int e0 = beg + 16 * part; e0 < end; e0 += 16 * wpr) {
+      const bool live = e0 + r < end;  // rows past the end: computed on the last edge, not stored
+      int e = min(e0 + r, end - 1), zr = 0, z0 = 0, z1 = 0;
+      if constexpr (MULTI) {
+        const int o = order[e];
+        e = beg + (o & 0xffffff), zr = o >> 24;
+        z0 = __builtin_amdgcn_readfirstlane(zr);
+        z1 = __builtin_amdgcn_readlane(zr, 15);  // the row is in species order
+      }
+      const float4 yv = ld4(Y + (int64_t)e * 16 + 4 * g);  // B: k = lm = 4g + s, column = edge r
+      f4v a1[4], a2[4], a3[4];
+      hidden_fwd_x<true, RND, NP>(swf, wi.w, live, e, nb, ef, a1, a2, a3, nullptr);
+      float h[16];  // B: k step (t, i): q = 16t + 4g + i, column = edge r
+#pragma unroll
+      for (int q = 0; q < 16; ++q) h[q] = qh(silu(a3[q >> 2][q & 3]), RND);
+      f4v gh[4], gy = f4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int t = 0; t < 4; ++t) gh[t] = f4v{0.f, 0.f, 0.f, 0.f};
+      for (int z = z0; z <= z1; ++z) {
+        const bool mine = !MULTI || zr == z;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          const float* row = gs + first_col(4 * g + s, z, kb) + r;
+          const float ym = mine ? comp(yv, s) : 0.f;
+#pragma unroll
+          for (int t = 0; t < 4; ++t) gh[t] = mfma16(row[16 * t], ym, gh[t]);
+        }
+        const float* row = gs + first_col(r, z, kb) + 4 * g;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const float4 w = ld4(row + 16 * t);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) gy = mfma16(comp(w, i), mine ? h[4 * t + i] : 0.f, gy);
+        }
+      }
+      float v[16];
+#pragma unroll
+      for (int q = 0; q < 16; ++q) v[q] = gh[q >> 2][q & 3];
+      const f4v o = hidden_vjp<true, RND, NP>(sw, wi, v, [&](int k, float* out) {
+        const f4v* a = k == 0 ? a1 : k == 1 ? a2 : a3;
+#pragma unroll
+        for (int q = 0; q < 16; ++q) out[q] = dsilu(a[q >> 2][q & 3]);
+      });
+      if (live) {
+        float4* dst = reinterpret_cast<float4*>(gY + (int64_t)e * gyp * 16 + 4 * g);
+        const float4 old = accumulate_gY ? *dst : float4{0.f, 0.f, 0.f, 0.f};
+        *dst = float4{old.x + gy[0], old.y + gy[1], old.z + gy[2], old.w + gy[3]};
+        store_gef(gef + (int64_t)e * nb, g, nb, o, accumulate);
+      }
+    }
+  }
+}
+
+// The first layer's folded weights F_l[z][q][v] = sum_u W3[q][l NC + u] x_z[u] Wl[u][v] (double
+// sums), one block per (q, z, l), as split fp16 planes scaled by s[l]: wf[l] = [hi | lo] of
+// [v][64 zi + q] (forward), wb[l] = [hi | lo] of [64 zi + q][v] (VJP).  amax (if given): instead of
+// writing planes, the largest |F_l| over the blocks, as float bits
+struct FirstFold {
+  const float* lin[4];
+  _Float16* wf[4];
+  _Float16* wb[4];
+  float s[4];
+};
+__global__ void __launch_bounds__(NC) k_first_fold(int W, int cout, const float* __restrict__ W3,
+                                                   const float* __restrict__ x, const int* __restrict__ present,
+                                                   int nz, FirstFold F, unsigned* __restrict__ amax) {
+  __shared__ double t[NC];
+  const int q = blockIdx.x, zi = blockIdx.y, lo = blockIdx.z, z = present ? present[zi] : zi;
+  t[threadIdx.x] = (double)W3[(int64_t)q * W + lo * NC + threadIdx.x] * x[(int64_t)z * NC + threadIdx.x];
+  __syncthreads();
+  const float* lin = F.lin[lo];
+  const int64_t K = 64 * (int64_t)nz, k = 64 * (int64_t)zi + q;
+  for (int v = threadIdx.x; v < cout; v += NC) {
+    double a = 0.0;
+    for (int u = 0; u < NC; ++u) a += t[u] * lin[(int64_t)u * cout + v];
+    if (amax) {
+      atomicMax(amax + lo, __float_as_uint(fabsf((float)a)));
+      continue;
+    }
+    const double xs = a * F.s[lo];
+    const _Float16 hi = (_Float16)(float)xs, low = (_Float16)(float)(xs - (double)(float)hi);
+    F.wf[lo][v * K + k] = hi;
+    F.wf[lo][(cout + v) * K + k] = low;
+    F.wb[lo][k * cout + v] = hi;
+    F.wb[lo][(K + k) * cout + v] = low;
   }
 }
 
@@ -1688,6 +1982,75 @@ void launch_mlp_hidden_bwd_x(hipStream_t st, int64_t E, int nb, const void* tile
   else
     MACE_HBX(RND_NONE);
 #undef MACE_HBX
+}
+
+void launch_first_order(hipStream_t st, int N, const int* rowptr, const int* sender, const int* species,
+                        const int* zslot, int nz, int* order) {
+  if (N <= 0) return;
+  MACE_LAUNCH(k_first_order, dim3(nblk(N, 4)), dim3(256), 0, st, N, rowptr, sender, species, zslot, nz, order);
+}
+
+void launch_first_fwd(hipStream_t st, int N, int nb, const int* rowptr, const float* ef, const float* Y,
+                      const int* order, int nz, int kb, const void* tiles, const float* winv3, float* S, int rnd) {
+  if (N <= 0) return;
+  MlpWinv wi{{winv3[0], winv3[1], winv3[2]}};
+  // as many blocks as fit at once (64 KB of LDS, 44 KB under the half policies)
+  const dim3 grid((unsigned)std::min(N, rnd == RND_NONE ? 512 : 768));
+#define MACE_FF(R, MU)                                                                                         \
+  MACE_LAUNCH((k_first_fwd<R, MU>), grid, dim3(256), 0, st, N, nb, rowptr, ef, Y, order, nz, kb,               \
+              static_cast<const MlpFwdX*>(tiles), wi, S)
+#define MACE_FFZ(R)               \
+  if (nz == 1) MACE_FF(R, false); \
+  else MACE_FF(R, true)
+  if (rnd == RND_F16) {
+    MACE_FFZ(RND_F16);
+  } else if (rnd == RND_BF16) {
+    MACE_FFZ(RND_BF16);
+  } else {
+    MACE_FFZ(RND_NONE);
+  }
+#undef MACE_FFZ
+#undef MACE_FF
+}
+
+void launch_first_bwd(hipStream_t st, int N, int nb, const int* rowptr, const float* ef, const float* Y,
+                      const int* order, int nz, int kb, const void* tiles, const float* winv3, const float* gS,
+                      float* gY, int gyp, int accumulate_gY, float* gef, int accumulate, int rnd) {
+  if (N <= 0) return;
+  MlpWinv wi{{winv3[0], winv3[1], winv3[2]}};
+  const MlpFwdX* fw = static_cast<const MlpFwdX*>(tiles);
+  const MlpBwdX* bw = reinterpret_cast<const MlpBwdX*>(static_cast<const char*>(tiles) + sizeof(MlpFwdX));
+  // waves per receiver: the fewest that give every SIMD two waves (2,048 on 256 CUs), at most four
+  int wl = 0;
+  while (wl < 2 && ((int64_t)N << wl) < 2048) ++wl;
+  // both tile images in LDS (76 KB, 38 KB under the half policies)
+  const dim3 grid((unsigned)std::min(((N << wl) + 3) / 4, rnd == RND_NONE ? 512 : 768));
+#define MACE_FB(R, MU)                                                                                              \
+  MACE_LAUNCH((k_first_bwd<R, MU>), grid, dim3(256), 0, st, N, wl, nb, rowptr, ef, Y, order, kb, fw, bw, wi, gS, gY, \
+              gyp, accumulate_gY, gef, accumulate)
+#define MACE_FBZ(R)               \
+  if (nz == 1) MACE_FB(R, false); \
+  else MACE_FB(R, true)
+  if (rnd == RND_F16) {
+    MACE_FBZ(RND_F16);
+  } else if (rnd == RND_BF16) {
+    MACE_FBZ(RND_BF16);
+  } else {
+    MACE_FBZ(RND_NONE);
+  }
+#undef MACE_FBZ
+#undef MACE_FB
+}
+
+void launch_first_fold(hipStream_t st, int W, int cout, const float* W3, const float* x, const int* present, int nz,
+                       const float* const* lin, _Float16* const* wf, _Float16* const* wb, const float* scale,
+                       unsigned* amax) {
+  FirstFold F{};
+  for (int lo = 0; lo < 4; ++lo) {
+    F.lin[lo] = lin[lo];
+    if (!amax) F.wf[lo] = wf[lo], F.wb[lo] = wb[lo], F.s[lo] = scale[lo];
+  }
+  MACE_LAUNCH(k_first_fold, dim3(64, nz, 4), dim3(NC), 0, st, W, cout, W3, x, present, nz, F, amax);
 }
 
 void launch_mlp_permute(hipStream_t st, int nb, const float* W0, const float* W1, const float* W2, void* tiles) {

@@ -129,8 +129,10 @@ __global__ void __launch_bounds__(256) k_gemm_group(GemmGroup G) {
 }
 
 // Float32 policy on fp16 matrix cores: the grouped products of k_gemm_group with
-// both operands split into fp16 pairs (a = a_hi + a_lo, three products per pair,
-// fp32 accumulation; about 2^-22 relative per product).  Roles are swapped: A =
+// both operands split into fp16 pairs (a = a_hi + a_lo, all four products per pair,
+// fp32 accumulation: what is lost is the splits' own residual, about 2^-23 per
+// operand; without lo x lo, which costs nothing here, the energies of the medium
+// model were three times further from float64, 4.0e-8 against 1.3e-8).  Roles are swapped: A =
 // weight rows (output columns), B = X^T with a tile's 16 rows as columns, so lane
 // (g, r) owns row r's eight k values of a 32-wide chunk and the accumulators of
 // that row: it scales the values by the power of two that maps their chunk's
@@ -255,8 +257,9 @@ __global__ void __launch_bounds__(256) k_gemm_group_x(GemmGroup G) {
           const int col = 16 * u + r;
           const h8 wh = *reinterpret_cast<const h8*>(&sW[buf][0][col][8 * g]);
           const h8 wl = *reinterpret_cast<const h8*>(&sW[buf][1][col][8 * g]);
-          f4v d = mfma16h(wl, xh, f4v{0.f, 0.f, 0.f, 0.f});
+          f4v d = mfma16h(wl, xl, f4v{0.f, 0.f, 0.f, 0.f});
           d = mfma16h(wh, xl, d);
+          d = mfma16h(wl, xh, d);
           d = mfma16h(wh, xh, d);
 #pragma unroll
           for (int i = 0; i < 4; ++i) acc[u][i] = fmaf(d[i], inv, acc[u][i]);
