@@ -2211,9 +2211,9 @@ void set_batch(mace_ctx* c, int32_t G, const int32_t* n_atoms, const int32_t* sp
     c->species.ensure(std::max(n, 1));
     if (n > 0) HIPCHK(hipMemcpy(c->species.p, species, (size_t)n * sizeof(int), hipMemcpyHostToDevice));
     c->first.order_valid = false;
-    if (first_sum(c, 0) && (!c->first.edges_for || (c->first.nz > 1 && c->first.order.n < (size_t)c->E)))
-      ensure_edge_buffers(c, c->E);
-    else if (!first_sum(c, 0) && c->first.edges_for)
+    // the current list's buffers in the layout of the path now taken (a new list allocates its own)
+    const bool sums = first_sum(c, 0);
+    if (c->E > 0 && (sums != c->first.edges_for || (sums && c->first.nz > 1 && c->first.order.n < (size_t)c->E)))
       ensure_edge_buffers(c, c->E);
     if (topo_changed || c->edges_manual) {  // a manual edge list lasts until the next set_system
       c->nl_valid = false;

@@ -1521,7 +1521,7 @@ __global__ void __launch_bounds__(256) k_first_bwd(int N, int wl, int nb, const 
 }
 
 // The first layer's folded weights F_l[z][q][v] = sum_u W3[q][l NC + u] x_z[u] Wl[u][v] (double
-// sums), one block per (q, z, l), as split fp16 planes scaled by s[l]: wf[l] = [hi | lo] of
+// sums), one block per (eight q, z, l), as split fp16 planes scaled by s[l]: wf[l] = [hi | lo] of
 // [v][64 zi + q] (forward), wb[l] = [hi | lo] of [64 zi + q][v] (VJP).  amax (if given): instead of
 // writing planes, the largest |F_l| over the blocks, as float bits
 struct FirstFold {
@@ -1530,28 +1530,44 @@ struct FirstFold {
   _Float16* wb[4];
   float s[4];
 };
+constexpr int kFoldQ = 8;  // q per block: each message-linear value read feeds eight sums
 __global__ void __launch_bounds__(NC) k_first_fold(int W, int cout, const float* __restrict__ W3,
                                                    const float* __restrict__ x, const int* __restrict__ present,
                                                    int nz, FirstFold F, unsigned* __restrict__ amax) {
-  __shared__ double t[NC];
-  const int q = blockIdx.x, zi = blockIdx.y, lo = blockIdx.z, z = present ? present[zi] : zi;
-  t[threadIdx.x] = (double)W3[(int64_t)q * W + lo * NC + threadIdx.x] * x[(int64_t)z * NC + threadIdx.x];
+  __shared__ double t[NC][kFoldQ];
+  const int q0 = blockIdx.x * kFoldQ, zi = blockIdx.y, lo = blockIdx.z, z = present ? present[zi] : zi;
+  const double xz = x[(int64_t)z * NC + threadIdx.x];
+#pragma unroll
+  for (int q = 0; q < kFoldQ; ++q)
+    t[threadIdx.x][q] = W3[(int64_t)(q0 + q) * W + lo * NC + threadIdx.x] * xz;
   __syncthreads();
   const float* lin = F.lin[lo];
-  const int64_t K = 64 * (int64_t)nz, k = 64 * (int64_t)zi + q;
+  const int64_t K = 64 * (int64_t)nz;
   for (int v = threadIdx.x; v < cout; v += NC) {
-    double a = 0.0;
-    for (int u = 0; u < NC; ++u) a += t[u] * lin[(int64_t)u * cout + v];
+    double a[kFoldQ] = {};
+#pragma unroll 16
+    for (int u = 0; u < NC; ++u) {
+      const double w = lin[(int64_t)u * cout + v];
+#pragma unroll
+      for (int q = 0; q < kFoldQ; ++q) a[q] += t[u][q] * w;
+    }
     if (amax) {
-      atomicMax(amax + lo, __float_as_uint(fabsf((float)a)));
+      float m = 0.f;
+#pragma unroll
+      for (int q = 0; q < kFoldQ; ++q) m = fmaxf(m, fabsf((float)a[q]));
+      atomicMax(amax + lo, __float_as_uint(m));
       continue;
     }
-    const double xs = a * F.s[lo];
-    const _Float16 hi = (_Float16)(float)xs, low = (_Float16)(float)(xs - (double)(float)hi);
-    F.wf[lo][v * K + k] = hi;
-    F.wf[lo][(cout + v) * K + k] = low;
-    F.wb[lo][k * cout + v] = hi;
-    F.wb[lo][(K + k) * cout + v] = low;
+#pragma unroll
+    for (int q = 0; q < kFoldQ; ++q) {
+      const int64_t k = 64 * (int64_t)zi + q0 + q;
+      const double xs = a[q] * F.s[lo];
+      const _Float16 hi = (_Float16)(float)xs, low = (_Float16)(float)(xs - (double)(float)hi);
+      F.wf[lo][v * K + k] = hi;
+      F.wf[lo][(cout + v) * K + k] = low;
+      F.wb[lo][k * cout + v] = hi;
+      F.wb[lo][(K + k) * cout + v] = low;
+    }
   }
 }
 
@@ -2050,7 +2066,7 @@ void launch_first_fold(hipStream_t st, int W, int cout, const float* W3, const f
     F.lin[lo] = lin[lo];
     if (!amax) F.wf[lo] = wf[lo], F.wb[lo] = wb[lo], F.s[lo] = scale[lo];
   }
-  MACE_LAUNCH(k_first_fold, dim3(64, nz, 4), dim3(NC), 0, st, W, cout, W3, x, present, nz, F, amax);
+  MACE_LAUNCH(k_first_fold, dim3(64 / kFoldQ, nz, 4), dim3(NC), 0, st, W, cout, W3, x, present, nz, F, amax);
 }
 
 void launch_mlp_permute(hipStream_t st, int nb, const float* W0, const float* W1, const float* W2, void* tiles) {
